@@ -1,0 +1,84 @@
+// bf3.hpp -- FP32 products on the bf16 matrix unit by exact splitting.
+//
+// An FP32 value is the sum of three bf16 values, x = h + m + l: h the top
+// eight significand bits (truncated), m the rest rounded to eight bits, l
+// what is left, which eight bits hold exactly (24 = 8 + 8 + 8; values whose
+// pieces would fall below 2^-126 lose those bits, an absolute error under
+// 2^-133).  A product a.b is then formed as six bf16 MFMAs, each exact into an FP32
+// accumulator:
+//   main   h.h
+//   cross  h.m + m.h + m.m + h.l + l.h
+// and the three dropped terms (m.l, l.m, l.l) are below 2^-23 of the product
+// with random signs.  v_mfma_f32_32x32x16_bf16 multiplies 16384 pairs in 32
+// cycles where v_mfma_f32_16x16x4_f32 takes 512: six of them are 2.7 times
+// the FP32 matrix rate.  Against 64 bits, sums of K products of N(0, 1)
+// values are off by (2-norm, MI355X): K = 64 5.4e-8, 768 1.6e-7, 6144 4.9e-7,
+// with FP32 MFMA 1.4e-7, 4.9e-7, 1.4e-6, the cross terms in an accumulator of
+// their own; with both in one accumulator 9.5e-8, 4.1e-7, 1.3e-6.
+//
+// Infinities and NaN: h keeps them (truncation never overflows), while m and
+// l become NaN and meet the cross accumulator only, so a non-finite main sum
+// is the result as it stands (bf3_join): the FP32 product's own value.
+#pragma once
+
+#include "common.hpp"
+
+namespace cxg {
+
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef float f16 __attribute__((ext_vector_type(16)));
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f16 mfma32b(b8 a, b8 b, f16 c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f4 mfma16b(b8 a, b8 b, f4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// The pieces of two values, each pair packed (a low, b high): eleven VALU
+// instructions.
+__device__ __forceinline__ void bf3_split2(float a, float b, unsigned& h, unsigned& m, unsigned& l)
+{
+    const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+    h = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+    const float ra = a - __builtin_bit_cast(float, ua & 0xffff0000u);
+    const float rb = b - __builtin_bit_cast(float, ub & 0xffff0000u);
+    m = __builtin_bit_cast(unsigned, __builtin_convertvector((f2){ra, rb}, b2));
+    const float sa = ra - __builtin_bit_cast(float, m << 16);
+    const float sb = rb - __builtin_bit_cast(float, m & 0xffff0000u);
+    l = __builtin_bit_cast(unsigned, __builtin_convertvector((f2){sa, sb}, b2));
+}
+
+// The same in four parts of two or three instructions, for a caller that puts
+// MFMAs between them: a and b are left as the rests.
+__device__ __forceinline__ void bf3_split2_part(int part, float& a, float& b, unsigned& h, unsigned& m,
+                                                unsigned& l)
+{
+    const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+    if (part == 0) {
+        h = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+        a -= __builtin_bit_cast(float, ua & 0xffff0000u);
+    } else if (part == 1) {
+        b -= __builtin_bit_cast(float, ub & 0xffff0000u);
+        m = __builtin_bit_cast(unsigned, __builtin_convertvector((f2){a, b}, b2));
+    } else if (part == 2) {
+        a -= __builtin_bit_cast(float, m << 16);
+    } else {
+        b -= __builtin_bit_cast(float, m & 0xffff0000u);
+        l = __builtin_bit_cast(unsigned, __builtin_convertvector((f2){a, b}, b2));
+    }
+}
+
+// A sum from its main and cross accumulators.
+__device__ __forceinline__ float bf3_join(float main, float cross)
+{
+    return __builtin_isfinite(main) ? main + cross : main;
+}
+
+} // namespace cxg
