@@ -41,6 +41,13 @@ __device__ __forceinline__ f4 mfma16b(b8 a, b8 b, f4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// A finished chain of MFMAs, before vector or memory instructions read it.  The
+// compiler's own wait for a 32x32x16 result has been seen four cycles short
+// where a branch lies between the MFMA and the reader (the last of the sixteen
+// registers came out stale), so the wait is written out: sixteen wait states,
+// where the matrix unit needs eleven.
+__device__ __forceinline__ void settle(f16& x) { asm volatile("s_nop 15" : "+v"(x)); }
+
 // The pieces of two values, each pair packed (a low, b high): eleven VALU
 // instructions.
 __device__ __forceinline__ void bf3_split2(float a, float b, unsigned& h, unsigned& m, unsigned& l)

@@ -378,6 +378,11 @@ __global__ __launch_bounds__(512, 2) void ffn_gemm_kernel(GemmArgs a)
         // columns wn + 32j + 8q + 4g .. +3.  A piece of a tile shared with
         // neighbouring runs goes to slot 0 if it opens this run, else slot 1
         // (then it closes the run).
+#pragma unroll
+        for (int q = 0; q < 2 * MI; q++) {
+            settle(acc[q >> 1][q & 1]);
+            settle(crs[q >> 1][q & 1]);
+        }
         const bool whole = ka == 0 && kb == a.KT;
         float* P = a.part + ((long)2 * blockIdx.x + (u == ub ? 0 : 1)) * (TM * GT);
 #pragma unroll

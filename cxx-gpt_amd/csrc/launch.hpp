@@ -97,6 +97,19 @@ hipError_t mha_nar_bwd_launch(const float* Q, const float* K, const float* V, co
                               const float* dO, const float* lse, float* dQ, float* dK, float* dV,
                               int B, int S, int H, int Dh, hipStream_t st,
                               const MhaRope* rope = nullptr);
+// The same attention with its products on split bf16 MFMAs (mhabf.hip): heads
+// of 17 .. 96 columns (a multiple of 4), 16-byte aligned tensors, no RoPE.
+// *_use: whether the shape is one where they are the faster.
+int mha_device_cus();
+bool mhabf_fwd_use(int B, int S, int H, int Dh, const float* Q, const float* K, const float* V,
+                   const float* O);
+bool mhabf_bwd_use(int B, int S, int H, int Dh, const float* Q, const float* K, const float* V,
+                   const float* dO, const float* dK, const float* dV);
+hipError_t mhabf_fwd_launch(const float* Q, const float* K, const float* V, float* O, float* lse,
+                            int B, int S, int H, int Dh, hipStream_t st);
+hipError_t mhabf_bwd_launch(const float* Q, const float* K, const float* V, const float* dO,
+                            const float* lse, const float* Di, float* dQ, float* dK, float* dV,
+                            int B, int S, int H, int Dh, hipStream_t st);
 hipError_t mha_bwd_prep_launch(const float* O, const float* dO, float* Di, float* dQ,
                                int B, int S, int H, int Dh, hipStream_t st);
 // lse (the statistics pass) and the pre-pass's Di and dQ = 0 in one launch, for

@@ -1355,7 +1355,7 @@ __global__ __launch_bounds__(256 * NSPLIT) void mha_bwd_kernel(
 static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Compute units of the current device (cached per device).
-static int device_cus()
+int mha_device_cus()
 {
     static int cached[64];
     int dev = 0;
@@ -1380,7 +1380,7 @@ static int device_cus()
 // Persistent workgroups also prefetch their next job.
 static unsigned job_grid(long njobs, int per_cu, bool even_rounds)
 {
-    const long g = (long)device_cus() * per_cu;
+    const long g = (long)mha_device_cus() * per_cu;
     const long rounds = (njobs + g - 1) / g;
     if (rounds <= 2 || (even_rounds && rounds % 2 == 0))
         return (unsigned)(njobs < g ? njobs : g);
@@ -1421,7 +1421,7 @@ static hipError_t fwd_dispatch2(const float* Q, const float* K, const float* V, 
     const int nqb = (S + MHA_BM - 1) / MHA_BM;
     const float qscale = (1.0f / sqrtf((float)Dh)) * kLog2e;
     const long njobs = (long)nqb * BH;
-    const int cus = device_cus();
+    const int cus = mha_device_cus();
     int pair = 0;
     dim3 grid(job_grid(njobs, MhaSplits<DHP>::FWD_PER_CU, false)), block(256 * NS);
     if (MhaSplits<DHP>::FWD_PAIR && njobs > cus && njobs <= 2L * cus) {
@@ -1492,6 +1492,8 @@ hipError_t mha_fwd_launch(const float* Q, const float* K, const float* V, float*
 {
     if (mha_nar_ok(B, S, H, Dh))
         return mha_nar_fwd_launch(Q, K, V, O, lse, B, S, H, Dh, st, rope);
+    if (rope == nullptr && mhabf_fwd_use(B, S, H, Dh, Q, K, V, O))
+        return mhabf_fwd_launch(Q, K, V, O, lse, B, S, H, Dh, st);
     if (Dh <= 16)
         return fwd_dispatch<16>(Q, K, V, O, lse, B, S, H, Dh, st, rope);
     if (Dh <= 32)
@@ -1511,7 +1513,7 @@ hipError_t mha_fwd_launch(const float* Q, const float* K, const float* V, float*
 bool mha_stats_prep_ok(int B, int S, int H, int Dh)
 {
     const long njobs = (long)B * H * ((S + MHA_BM - 1) / MHA_BM);
-    return Dh <= 64 && njobs <= 2L * device_cus();
+    return Dh <= 64 && njobs <= 2L * mha_device_cus();
 }
 
 // Statistics pass (lse) with the backward's pre-pass (Di, dQ = 0) in the same
@@ -1726,8 +1728,10 @@ bool mha_bwd_iprep_ok(int B, int S, int H, int Dh, const float* Q, const float* 
     if (!aligned16(Q) || !aligned16(K) || !aligned16(V) || !aligned16(dO) || !aligned16(O) ||
         !aligned16(dQ) || !aligned16(dK) || !aligned16(dV))
         return false;
+    if (mhabf_bwd_use(B, S, H, Dh, Q, K, V, dO, dK, dV))
+        return false;   // its kernel takes Di and a zeroed dQ
     const long njobs = (long)((S + MHA_BN - 1) / MHA_BN) * B * H;
-    const long slots = (long)device_cus() * bwd_per_cu<64, false>();
+    const long slots = (long)mha_device_cus() * bwd_per_cu<64, false>();
     return (long)job_grid(njobs, bwd_per_cu<64, false>(), true) <= slots;
 }
 
@@ -1740,6 +1744,8 @@ hipError_t mha_bwd_main_launch(const float* Q, const float* K, const float* V, c
     const MhaRope& rp = rope != nullptr ? *rope : none;
     if (ip != nullptr && (rope != nullptr || Dh != 64))
         return hipErrorInvalidValue;
+    if (rope == nullptr && ip == nullptr && mhabf_bwd_use(B, S, H, Dh, Q, K, V, dO, dK, dV))
+        return mhabf_bwd_launch(Q, K, V, dO, lse, Di, dQ, dK, dV, B, S, H, Dh, st);
 #define CXG_BWD(D)                                                                            \
     return rope != nullptr                                                                    \
                ? bwd_dispatch<D, true>(Q, K, V, dO, lse, Di, dQ, dK, dV, B, S, H, Dh, st, rp,  \

@@ -71,3 +71,84 @@ def test_ffn_non_finite(dev, M, E, F):
     inf = torch.isinf(want) & ~big | torch.isinf(X.double() @ W1.double().t())
     assert torch.equal(pre[inf], want[inf])
     assert bool(torch.isfinite(pre[torch.isfinite(want) & ~big]).all())
+
+
+def heads(t, B, S, H, Dh):
+    return t.double().view(B, S, H, Dh).permute(0, 2, 1, 3).reshape(B * H, S, Dh)
+
+
+def flat(t, B, S, H, Dh):
+    return t.view(B, H, S, Dh).permute(0, 2, 1, 3).reshape(B * S, H * Dh)
+
+
+def mha64(Q, K, V, dO, B, S, H, Dh):
+    """float64 causal attention, its row statistics and gradients, and a bound
+    on each one's FP32 error: a score q.k is off by at most (Dh / 8 + 16) 2^-24
+    of sum |q||k| (gemm_bound), lse by as much, so P by twice that relatively
+    (plus the exponential's 2^-22), and the sums over rows by (S / 8 + 16) 2^-24
+    of their terms' magnitudes."""
+    q, k, v, do = (heads(t, B, S, H, Dh) for t in (Q, K, V, dO))
+    T = lambda t: t.transpose(1, 2).contiguous()   # noqa: E731
+    scale = Dh ** -0.5
+    future = torch.ones(S, S, device=q.device, dtype=torch.bool).triu_(1)
+    s = (torch.bmm(q, T(k)) * scale).masked_fill_(future, -np.inf)
+    lse = torch.logsumexp(s, 2)
+    p = torch.exp(s - lse.unsqueeze(2))
+    o = torch.bmm(p, v)
+    di = (do * o).sum(2, keepdim=True)
+    ds = (torch.bmm(do, T(v)) - di) * p * scale
+    out = [o, torch.bmm(ds, k), torch.bmm(T(ds), q), torch.bmm(T(p), do)]
+    es = (Dh / 8 + 16) * 2.0 ** -24 * (torch.bmm(q.abs(), T(k.abs())) * scale).masked_fill_(future, 0)
+    e = 2 * es.amax(2, keepdim=True) + 2.0 ** -22 + (S / 8 + 16) * 2.0 ** -24
+    pe = p * e
+    we = p * (torch.bmm(do.abs(), T(v.abs())) + (do * o).abs().sum(2, keepdim=True)) * scale * e * 2
+    lim = [torch.bmm(pe, v.abs()), torch.bmm(we, k.abs()), torch.bmm(T(we), q.abs()),
+           torch.bmm(T(pe), do.abs())]
+    return ([flat(t, B, S, H, Dh) for t in out] + [lse],
+            [flat(t, B, S, H, Dh) for t in lim] + [e.squeeze(2)])
+
+
+def within(got, want, lim, name):
+    err = (got.double() - want).abs() / (lim + 1e-12)
+    assert bool(torch.isfinite(got).all()) and err.max().item() <= 1.0, f"{name}: {err.max().item()}"
+
+
+# (B, S, H, Dh): each kernel at the edges of its 32- and 64-row tiles, of its
+# column steps (Dh 20 .. 96) and of its rule (64-row tiles against 256 units):
+# one round, one to two, many; rows past S in the last tile
+@pytest.mark.parametrize("B,S,H,Dh", [
+    (2, 96, 3, 20), (1, 127, 4, 32), (3, 161, 2, 36), (1, 128, 5, 64), (2, 321, 3, 64),
+    (2, 65, 2, 68), (1, 333, 3, 80), (2, 31, 2, 96), (1, 193, 4, 92),
+    (8, 300, 8, 64), (8, 257, 15, 36), (16, 257, 9, 64), (16, 290, 8, 24)])
+@pytest.mark.parametrize("use_lse", [True, False])
+def test_mha_split(dev, B, S, H, Dh, use_lse):
+    g = torch.Generator(device=dev).manual_seed(S * Dh)
+    Q, K, V, dO = (torch.randn(B * S, H * Dh, device=dev, generator=g) for _ in range(4))
+    Q[: S // 2] *= 6.0   # scores that move the softmax reference between tiles
+    O, dQ, dK, dV = (torch.full_like(Q, np.nan) for _ in range(4))
+    lse = torch.empty(B * H, S, device=dev) if use_lse else None
+    cx.mha_fwd(Q, K, V, O, B, S, H, Dh, lse=lse)
+    cx.mha_bwd(Q, K, V, O, dO, dQ, dK, dV, B, S, H, Dh, lse=lse)
+    want, lim = mha64(Q, K, V, dO, B, S, H, Dh)
+    for got, w, e, n in zip((O, dQ, dK, dV, lse), want, lim, ("O", "dQ", "dK", "dV", "lse")):
+        if got is not None:
+            within(got, w, e, n)
+
+
+@pytest.mark.parametrize("B,S,H,Dh", [(1, 160, 2, 64), (1, 100, 2, 96), (16, 257, 9, 64)])
+def test_mha_minus_infinite_scores(dev, B, S, H, Dh):
+    """A key whose scores are all -inf has probability 0, as in FP32."""
+    g = torch.Generator(device=dev).manual_seed(9)
+    Q, K, V = (torch.randn(B * S, H * Dh, device=dev, generator=g) for _ in range(3))
+    Q[:, 0] = Q[:, 0].abs() + 0.5
+    K.view(B, S, -1)[:, 3::7, 0] = -np.inf   # head 0; never a sequence's first key
+    O = torch.empty_like(Q)
+    cx.mha_fwd(Q, K, V, O, B, S, H, Dh)
+    fin = K.clamp(min=-1e3)   # scores below -60 of the others': probability 0 to FP32 as well
+    want, lim = mha64(Q, fin, V, V, B, S, H, Dh)
+    rows = heads(K, B, S, H, Dh).isfinite().all(2, keepdim=True)
+    assert bool(torch.isfinite(O).all())
+    # the bound of the same products without the infinite keys
+    lim = mha64(Q, torch.where(flat(rows.expand(-1, -1, Dh), B, S, H, Dh), K, torch.zeros_like(K)), V, V,
+                B, S, H, Dh)[1]
+    within(O, want[0], lim[0] * 4, "O")
