@@ -123,22 +123,30 @@ def missing_symbols():
 
 
 def _ptr(t):
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()   # argtypes make it a void*
+
+
+_torch_stream = None
 
 
 def _stream(stream):
     if stream is not None:
-        return ctypes.c_void_p(stream)
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return stream
+    global _torch_stream
+    if _torch_stream is None:
+        import torch
+        # the raw handle of the current device's current stream, without the
+        # Stream object that torch.cuda.current_stream() makes
+        raw, dev = torch._C._cuda_getCurrentRawStream, torch.cuda.current_device
+        _torch_stream = lambda: raw(dev())   # noqa: E731
+    return _torch_stream()
 
 
 def _call(name, *args):
-    st = getattr(lib(), name)(*args)
+    L = _lib if _lib is not None else lib()
+    st = getattr(L, name)(*args)
     if st != CXG_OK:
-        raise CxgError(name, st, lib().cxg_last_hip_error())
+        raise CxgError(name, st, L.cxg_last_hip_error())
     return st
 
 
