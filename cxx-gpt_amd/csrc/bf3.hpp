@@ -88,4 +88,80 @@ __device__ __forceinline__ float bf3_join(float main, float cross)
     return __builtin_isfinite(main) ? main + cross : main;
 }
 
+// LDS planes of bf16 rows, DHP columns a row.  A row's 16-byte chunks are
+// exchanged by its number, so that a row operand's ds_read_b128 and a column
+// operand's transposing read each cover the 64 banks once: measured, a wave's
+// b128 read takes 4.5 cycles so and 8 to 16 otherwise.
+template <int DHP>
+__device__ __forceinline__ int swz(int row)
+{
+    if constexpr (DHP == 32 || DHP == 96)
+        return (row >> 2) & 3;
+    else if constexpr (DHP == 64)
+        return 4 * ((row >> 1) & 1) + ((row >> 2) & 3);
+    else
+        return 4 * (row & 3) + ((row >> 2) & 3);
+}
+
+template <int DHP>
+__device__ __forceinline__ int chunk_off(int row, int c)
+{
+    return row * (DHP * 2) + ((c ^ swz<DHP>(row)) << 4);
+}
+
+// Column operand of k-step rows r0 .. r0+15 (r0 a multiple of 16), columns
+// c0 .. c0+31, from one plane: two transposing reads (ds_read_b64_tr_b16: a
+// group of 16 lanes reads four rows' 16 columns, lane i receiving column i).
+// Slot (g, e) is row r0 + 8 (e / 4) + 4g + e % 4, an accumulator's order, or
+// with NAT row r0 + 8g + e, a row operand's.
+template <int DHP, bool NAT = false>
+__device__ __forceinline__ b8 read_tr(const char* plane, int r0, int c0, int lane)
+{
+    typedef short s4v __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s4v* lp;
+    const int g = lane >> 5, i = lane & 15;
+    const int row = r0 + (NAT ? 8 : 4) * g + (i >> 2);
+    const int col = c0 + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
+    const char* a = plane + chunk_off<DHP>(row, col >> 3) + 2 * (col & 7);
+    const char* b = plane + chunk_off<DHP>(row + (NAT ? 4 : 8), col >> 3) + 2 * (col & 7);
+    const s4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)a);
+    const s4v y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)b);
+    return __builtin_bit_cast(b8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int DHP>
+__device__ __forceinline__ b8 read_row(const char* plane, int row, int c)
+{
+    return *reinterpret_cast<const b8*>(plane + chunk_off<DHP>(row, c));
+}
+
+// eight values to their three pieces
+__device__ __forceinline__ void split8(const float* v, b8& h, b8& m, b8& l)
+{
+    u4 x, y, z;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        unsigned a, b, c;
+        bf3_split2(v[2 * e], v[2 * e + 1], a, b, c);
+        x[e] = a;
+        y[e] = b;
+        z[e] = c;
+    }
+    h = __builtin_bit_cast(b8, x);
+    m = __builtin_bit_cast(b8, y);
+    l = __builtin_bit_cast(b8, z);
+}
+
+// The cross terms of a product: pieces (pa, pb) = h.m, m.h, m.m, h.l, l.h.
+constexpr int kPa[5] = {0, 1, 1, 0, 2}, kPb[5] = {1, 0, 1, 2, 0};
+
+__device__ __forceinline__ f16 f16zero()
+{
+    f16 z;
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+        z[i] = 0.0f;
+    return z;
+}
+
 } // namespace cxg

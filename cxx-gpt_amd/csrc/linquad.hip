@@ -30,6 +30,7 @@
 // Scratch: B' * nb(nb+1)/2 blocks of 256 floats per score matrix (nb =
 // ceil(S/16)) and the features; the path is taken when that fits
 // kQsBudget.
+#include "bf3.hpp"
 #include "common.hpp"
 #include "launch.hpp"
 #include "linattn.hpp"
@@ -588,6 +589,217 @@ __global__ __launch_bounds__(256) void lin_qs_prod_kernel(const QsArgs a,
 }
 
 // ---------------------------------------------------------------------------
+// phase 2 for launches that fill the chip (qs_tiles), on split bf16 MFMAs
+// (bf3.hpp): a workgroup of 4 waves forms a 64 x 64 tile of one output of one
+// sequence over 32-row steps of the other side.  A step's rows of X (V, phi(K),
+// phi(Q) or dnum) and its eight 16x16 score blocks go through LDS, split there
+// once for the 64 rows and columns that use them (the waves above load them
+// again for every 16 rows); X is read as column operand, the scores as rows (O,
+// dQ) or as columns (dK, dV) of the same planes.  Wave w: rows 32 (w / 2),
+// columns 32 (w % 2) of the tile; results transposed (X^T S^T), so a lane holds
+// 16-byte pieces of its own row.  Bound by a step's chain (loads two steps
+// ahead, split, barrier, LDS, twelve MFMAs, barrier: about 1 us) and hidden by
+// four workgroups a compute unit; 128-column tiles (two a unit), and two LDS
+// stages (three), were slower at every shape.  Kernel times, one wave a 16-row
+// unit -> tiles: 32 x S256, D = E = 512: gradients 54.8 -> 43.3 us, O 19.2 ->
+// 15.6; 32 x S384, 640: 156 -> 95.5, 50.8 -> 35.1; 8 x S256, 512: gradients
+// 18.9 -> 15.2.
+// ---------------------------------------------------------------------------
+template <int PHI, bool BWD>
+__global__ __launch_bounds__(256) void lin_qs_tile_kernel(const QsArgs a,
+                                                             const LinRopeArg<PHI> rope)
+{
+    constexpr int PX = 32 * 64 * 2, PSB = 64 * 32 * 2;   // bytes of a plane
+    __shared__ __attribute__((aligned(16))) char lds[3 * PX + 3 * PSB];
+    __shared__ float dsum[64][4];
+    __shared__ float rope_w[phi_rope(PHI) ? LIN_ROPE_MAX_D / 2 : 1];
+    rope_tab_lds<PHI, LIN_ROPE_MAX_D / 2>(rope_w, rope);
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, g = lane >> 5;
+    const int wr = w >> 1, wc = w & 1;
+
+    // heaviest first: job = (nrb - L) * units + unit for L 64-row blocks of steps
+    const int nrb = (a.S + 63) / 64;
+    const int nsD = a.nslD;
+    int seq, job;
+    if (!qs_xcd_job((int)blockIdx.x, a.Bq, nrb * a.units, seq, job))
+        return;   // the whole workgroup
+    const int L = nrb - job / a.units;
+    int kind, sl = job % a.units;
+    if (!BWD) {
+        kind = QS_O;
+    } else {
+        kind = QS_DQ;
+        if (!(a.kinds & 2) || sl >= nsD) {
+            sl -= (a.kinds & 2) ? nsD : 0;
+            kind = sl < nsD ? QS_DK : QS_DV;
+            sl -= sl < nsD ? 0 : nsD;
+        }
+    }
+    const bool qside = kind == QS_O || kind == QS_DQ;
+    const int blk = qside ? L - 1 : nrb - L, r0 = 64 * blk;   // the tile's first row
+    const int W = (kind == QS_O || kind == QS_DV) ? a.E : a.D;
+    const float* X = kind == QS_O ? a.V : kind == QS_DK ? a.Fq : kind == QS_DV ? a.dnum : a.Fk;
+    const float* Sb = (kind == QS_O || kind == QS_DV) ? a.Ab : a.Gb;
+    const long rb = (long)seq * a.S;
+    const int c0 = 64 * sl;
+    const __amdgpu_buffer_rsrc_t bx = qs_rows(X, rb, a.S, W);
+    const float* sbase = Sb + (long)seq * a.npairs * 256;
+    // steps: key rows 0 .. r0 + 63 (query side), query rows r0 .. S - 1
+    const int first = qside ? 0 : r0, last = qside ? min(r0 + 64, a.S) : a.S;
+    const int nk = (last - first + 31) / 32;
+
+    // this thread's share of a step: an eight-column chunk of X and eight floats of
+    // one row of score block (bi, bj): query side blocks 4 x 2, key side 2 x 4
+    unsigned xo[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int c = c0 + 8 * (tid & 7) + 4 * q;
+        xo[q] = c < W ? (unsigned)((tid >> 3) * W + c) * 4u : kDropOffset;
+    }
+    const int sblk = tid >> 5, srow = (tid & 31) >> 1, half = tid & 1;
+    const int bi = qside ? sblk >> 1 : sblk >> 2, bj = qside ? sblk & 1 : sblk & 3;
+    float xs2[2][8], sv2[2][8];   // two steps in flight: step n in set n % 2
+    auto load = [&](int n, auto set) {
+        auto& xv = xs2[decltype(set)::value];
+        auto& sv = sv2[decltype(set)::value];
+        const int k0 = first + 32 * n;
+        const unsigned so = (unsigned)(k0 * W) * 4u;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const f4 x = buffer_load_f4s(bx, xo[q], so);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                xv[4 * q + e] = x[e];
+        }
+        const int i = (qside ? r0 : k0) / 16 + bi, j = (qside ? k0 : r0) / 16 + bj;
+        const bool ok = j <= i && i < a.nb;   // else above the diagonal or past S
+        const float* sp = sbase + (ok ? (long)(i * (i + 1) / 2 + j) * 256 + srow * 16 + 8 * half : 0);
+        const f4 x = *reinterpret_cast<const f4*>(sp), y = *reinterpret_cast<const f4*>(sp + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            sv[e] = ok ? x[e] : 0.0f;
+            sv[4 + e] = ok ? y[e] : 0.0f;
+        }
+    };
+    float dp = 0.0f;   // O: this thread's part of its row's sum of A
+    char* const LS = lds + 3 * PX;
+    const int xat = chunk_off<64>(tid >> 3, tid & 7);
+    const int sat = qside ? chunk_off<32>(16 * bi + srow, 2 * bj + half)
+                          : chunk_off<64>(16 * bi + srow, 2 * bj + half);
+    auto put = [&](auto set) {
+        const auto& xv = xs2[decltype(set)::value];
+        const auto& sv = sv2[decltype(set)::value];
+        b8 h, m, l;
+        split8(xv, h, m, l);
+        *reinterpret_cast<b8*>(lds + xat) = h;
+        *reinterpret_cast<b8*>(lds + PX + xat) = m;
+        *reinterpret_cast<b8*>(lds + 2 * PX + xat) = l;
+        split8(sv, h, m, l);
+        *reinterpret_cast<b8*>(LS + sat) = h;
+        *reinterpret_cast<b8*>(LS + PSB + sat) = m;
+        *reinterpret_cast<b8*>(LS + 2 * PSB + sat) = l;
+        dp += ((sv[0] + sv[1]) + (sv[2] + sv[3])) + ((sv[4] + sv[5]) + (sv[6] + sv[7]));
+    };
+    f16 acc = f16zero(), crs = f16zero();
+    auto step = [&](int n, auto set) {
+        put(set);
+        __syncthreads();
+        if (n + 2 < nk)
+            load(n + 2, set);
+        // the step's blocks that reach this wave's rows
+        const int k0 = first + 32 * n, mine = r0 + 32 * wr;
+        if (qside ? k0 <= mine : k0 >= mine) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                b8 fs[3];
+#pragma unroll
+                for (int p = 0; p < 3; p++)
+                    fs[p] = qside ? read_row<32>(LS + p * PSB, 32 * wr + l32, 2 * t + g)
+                                  : read_tr<64, true>(LS + p * PSB, 16 * t, 32 * wr, lane);
+                b8 fx[3];
+#pragma unroll
+                for (int p = 0; p < 3; p++)
+                    fx[p] = read_tr<64, true>(lds + p * PX, 16 * t, 32 * wc, lane);
+                acc = mfma32b(fx[0], fs[0], acc);
+#pragma unroll
+                for (int x = 0; x < 5; x++)
+                    crs = mfma32b(fx[kPa[x]], fs[kPb[x]], crs);
+            }
+        }
+        __syncthreads();
+    };
+    load(0, ic<0>{});
+    if (nk > 1)
+        load(1, ic<1>{});
+    for (int n = 0; n < nk; n += 2) {
+        step(n, ic<0>{});
+        if (n + 1 < nk)
+            step(n + 1, ic<1>{});
+    }
+    settle(acc);
+    settle(crs);
+
+    // lane: row r0 + 32 wr + l32; piece q: columns c0 + 32 wc + 8q + 4g .. +3
+    const int row = r0 + 32 * wr + l32;
+    float inv = 1.0f;
+    if (kind == QS_O && a.norm) {
+        dsum[16 * bi + srow][2 * bj + half] = dp;
+        __syncthreads();
+        const float* d4 = dsum[32 * wr + l32];
+        const float d = (d4[0] + d4[1]) + (d4[2] + d4[3]);
+        inv = 1.0f / (d + 1e-8f);
+        if (row < a.S && sl == 0 && wc == 0 && g == 0)
+            a.den[rb + row] = a.den_eps ? d + 1e-8f : d;
+    }
+    if (row >= a.S)
+        return;
+    auto col = [&](int q) { return c0 + 32 * wc + 8 * q + 4 * g; };
+    auto piece = [&](int q) {
+        f4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            v[e] = bf3_join(acc[4 * q + e], crs[4 * q + e]);
+        return v;
+    };
+    if (kind == QS_O || kind == QS_DV) {
+        float* orow = (kind == QS_O ? a.O : a.dV) + (rb + row) * a.E;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (col(q) < a.E)
+                *reinterpret_cast<f4*>(orow + col(q)) = piece(q) * inv;
+        return;
+    }
+    // dQ, dK: phi' as in lin_qs_prod_kernel
+    float* orow = (kind == QS_DQ ? a.dQ : a.dK) + (rb + row) * a.D;
+    const float* raw = kind == QS_DQ ? a.Qx : a.Kx;
+    const float* fea = kind == QS_DQ ? a.Fq : a.Fk;
+    const bool from_f = !phi_rope(PHI) && fea != raw;
+    const float* xrow = (from_f ? fea : raw) + (rb + row) * a.D;
+    f4 xe[4];
+    if (PHI != PHI_NONE) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            xe[q] = *reinterpret_cast<const f4*>(xrow + min(col(q), a.D - 4));
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int c = col(q);
+        if (c >= a.D)
+            continue;
+        f4 v = piece(q);
+        if constexpr (phi_rope(PHI)) {
+            v = rope_phi_grad4<PHI>(v, xe[q], row, c, rope_w);
+        } else if constexpr (PHI != PHI_NONE) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                v[e] *= from_f ? Phi<PHI>::d_from_f(xe[q][e]) : Phi<PHI>::d(xe[q][e]);
+        }
+        *reinterpret_cast<f4*>(orow + c) = v;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 static size_t qs_al(size_t b) { return (b + 255) / 256 * 256; }
@@ -749,12 +961,30 @@ static int qs_split(const QsArgs& a, bool bwd)
     return units >= want ? 1 : 2 * units >= want ? 2 : 4;
 }
 
+// Whether the products run as 64 x 64 tiles: where these fill the chip, more
+// than two a compute unit forward, one and a half backward (whose old units are
+// the longer ones); with fewer, a tile's serial steps show and 16-row units
+// split over waves are faster (8 x S256, 512 forward, 256 tiles: 8.8 / 11.4 us;
+// 4 x S256, 512 backward, 384 tiles: 11.3 / 12.6; 10 x S190, 304 with the
+// rotation backward, 450 tiles: 20.7 / 11.6).
+static bool qs_tiles(const QsArgs& a, bool bwd)
+{
+    const long tiles = (long)a.Bq * ((a.S + 63) / 64) * a.units, cus = qs_cus();
+    return 2 * tiles > (bwd ? 3 : 4) * cus;
+}
+
 template <int PHI, bool BWD>
 static void qs_prod(const QsArgs& a, int D, hipStream_t st)
 {
     ProfScope ps(st, a.norm ? (BWD ? "lin_qs_grad" : "lin_qs_out")
                             : (BWD ? "gpt_qs_grad" : "gpt_qs_out"));
     const LinRopeArg<PHI> rope = lin_rope_arg<PHI>(D);
+    if (qs_tiles(a, BWD)) {
+        const long nrb = (a.S + 63) / 64;
+        CXG_LAUNCH((lin_qs_tile_kernel<PHI, BWD>), dim3(qs_grid(a.Bq, nrb * a.units)), dim3(256), 0,
+                   st, a, rope);
+        return;
+    }
     const int split = qs_split(a, BWD), upw = 4 / split;
     CXG_LAUNCH((lin_qs_prod_kernel<PHI, BWD>),
                dim3(qs_grid(a.Bq, (long)a.nb * ((a.units + upw - 1) / upw))), dim3(256), 0, st, a,

@@ -1,20 +1,16 @@
 // mhabf.hip -- causal softmax multi-head attention with its FP32 products on
 // the bf16 matrix unit (split operands, bf3.hpp).
 //
-// The same functions as mha.hip's tile kernels for heads of 17 to 128 columns
+// The same functions as mha.hip's tile kernels for heads of 17 to 96 columns
 // (16-byte aligned rows, no RoPE); mha.hip's dispatch says which shapes come
 // here.  Tensors (B*S, H*Dh) row-major, head h of row r at [(r*H + h)*Dh, +Dh);
 // lse, Di [B*H][S].
 //
 // LDS.  A streamed tile (K and V rows forward, Q and dO rows backward) is split
 // once, on its way from registers to LDS, into three planes of bf16 rows.  Each
-// plane serves both as a product's row operand (a lane reads eight consecutive
-// columns of its row, ds_read_b128) and, through the transposing read
-// (ds_read_b64_tr_b16: a group of 16 lanes reads four rows' 16 columns, lane i
-// receiving column i), as its column operand, so no second, transposed copy is
-// formed.  A row's 16-byte chunks are exchanged by its number (swz) so that
-// both kinds of read cover the 64 banks once: measured, a b128 read of a wave
-// takes 4.5 cycles so and 8 to 16 otherwise.
+// plane serves both as a product's row operand and, through the transposing
+// read, as its column operand (bf3.hpp), so no second, transposed copy is
+// formed.
 //
 // MFMA 32x32x16: lane (l32 = l % 32, g = l / 32) holds A[l32][8g + e], B[8g + e]
 // [l32] and D[8 (r / 4) + 4g + r % 4][l32].  A score accumulator's registers
@@ -29,80 +25,8 @@
 
 namespace cxg {
 
-typedef short s4v __attribute__((ext_vector_type(4)));
-typedef short s8v __attribute__((ext_vector_type(8)));
-
 constexpr float kLazy = 8.0f;   // log2 units a score may exceed its row's reference by
 constexpr float kBig = 3.0e38f;
-
-// rows of DHP bf16
-template <int DHP>
-__device__ __forceinline__ int swz(int row)
-{
-    if constexpr (DHP == 32 || DHP == 96)
-        return (row >> 2) & 3;
-    else if constexpr (DHP == 64)
-        return 4 * ((row >> 1) & 1) + ((row >> 2) & 3);
-    else
-        return 4 * (row & 3) + ((row >> 2) & 3);
-}
-
-template <int DHP>
-__device__ __forceinline__ int chunk_off(int row, int c)
-{
-    return row * (DHP * 2) + ((c ^ swz<DHP>(row)) << 4);
-}
-
-// Column operand of k-step rows r0 .. r0+15 (r0 a multiple of 16), columns
-// c0 .. c0+31, from one plane: two transposing reads.
-template <int DHP>
-__device__ __forceinline__ b8 read_tr(const char* plane, int r0, int c0, int lane)
-{
-    typedef __attribute__((address_space(3))) s4v* lp;
-    const int g = lane >> 5, i = lane & 15;
-    const int row = r0 + 4 * g + (i >> 2);
-    const int col = c0 + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
-    const char* a = plane + chunk_off<DHP>(row, col >> 3) + 2 * (col & 7);
-    const char* b = plane + chunk_off<DHP>(row + 8, col >> 3) + 2 * (col & 7);
-    const s4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)a);
-    const s4v y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)b);
-    return __builtin_bit_cast(b8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-template <int DHP>
-__device__ __forceinline__ b8 read_row(const char* plane, int row, int c)
-{
-    return *reinterpret_cast<const b8*>(plane + chunk_off<DHP>(row, c));
-}
-
-// eight values to their three pieces
-__device__ __forceinline__ void split8(const float* v, b8& h, b8& m, b8& l)
-{
-    u4 x, y, z;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        unsigned a, b, c;
-        bf3_split2(v[2 * e], v[2 * e + 1], a, b, c);
-        x[e] = a;
-        y[e] = b;
-        z[e] = c;
-    }
-    h = __builtin_bit_cast(b8, x);
-    m = __builtin_bit_cast(b8, y);
-    l = __builtin_bit_cast(b8, z);
-}
-
-// The cross terms of a product: pieces (pa, pb) = h.m, m.h, m.m, h.l, l.h.
-constexpr int kPa[5] = {0, 1, 1, 0, 2}, kPb[5] = {1, 0, 1, 2, 0};
-
-__device__ __forceinline__ f16 f16zero()
-{
-    f16 z;
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-        z[i] = 0.0f;
-    return z;
-}
 
 // A cross sum that an infinity or NaN in an operand has made NaN: any finite
 // value, since the main sum is then not finite and stands (bf3.hpp).

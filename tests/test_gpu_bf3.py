@@ -152,3 +152,65 @@ def test_mha_minus_infinite_scores(dev, B, S, H, Dh):
     lim = mha64(Q, torch.where(flat(rows.expand(-1, -1, Dh), B, S, H, Dh), K, torch.zeros_like(K)), V, V,
                 B, S, H, Dh)[1]
     within(O, want[0], lim[0] * 4, "O")
+
+
+# enough 64 x 64 tiles for the split products (more than 512 forward, 384
+# backward), at row, key-step and column remainders; with and without the
+# context, and the rotation
+@pytest.mark.parametrize("B,S,D,E", [(65, 65, 80, 112), (24, 190, 208, 208), (90, 33, 352, 144)])
+@pytest.mark.parametrize("api", ["kattn", "lin_elu", "rope"])
+def test_linear_tiles(dev, B, S, D, E, api):
+    if api == "lin_elu" and D != E:
+        pytest.skip("one width")
+    g = torch.Generator(device=dev).manual_seed(B + S)
+    Q, K = (torch.randn(B * S, D, device=dev, generator=g) for _ in range(2))
+    V, dO = (torch.randn(B * S, E, device=dev, generator=g) for _ in range(2))
+    O, dV = torch.full_like(V, np.nan), torch.full_like(V, np.nan)
+    dQ, dK = torch.full_like(Q, np.nan), torch.full_like(Q, np.nan)
+    den = torch.empty(B * S, device=dev)
+    n = cx.lin_ctx_size(B, S, D, E)
+    ctx = torch.empty(n // 4, device=dev) if n else None
+    q, k = (t.double().view(B, S, D) for t in (Q, K))
+    if api == "rope":
+        w = torch.tensor([10000.0 ** (-2 * i / D) for i in range(D // 2)], device=dev)
+        a = (torch.arange(S, device=dev).float()[:, None] * w).double()
+
+        def rot(x, s):
+            y = torch.empty_like(x)
+            c, t = torch.cos(a), s * torch.sin(a)
+            y[..., 0::2] = x[..., 0::2] * c - x[..., 1::2] * t
+            y[..., 1::2] = x[..., 0::2] * t + x[..., 1::2] * c
+            return y
+        q, k = rot(q, 1), rot(k, 1)
+        cx.kattn_rope_fwd(Q, K, V, O, den, B, S, D, E, ctx=ctx)
+        cx.kattn_rope_bwd(Q, K, V, O, dO, den, dQ, dK, dV, B, S, D, E, ctx=ctx)
+    elif api == "kattn":
+        cx.kattn_fwd(Q, K, V, O, den, None, None, None, B, S, D, E)
+        cx.kattn_bwd(Q, K, V, O, dO, den, dQ, dK, dV, B, S, D, E)
+    else:
+        cx.lin_elu_fwd(Q, K, V, O, den, ctx, B, S, E)
+        cx.lin_elu_bwd(Q, K, V, O, dO, den, dQ, dK, dV, B, S, E, ctx=ctx)
+    T = lambda t: t.transpose(1, 2).contiguous()   # noqa: E731
+    fq, fk = (torch.where(x > 0, x + 1, torch.exp(x)) for x in (q, k))
+    v, do = V.double().view(B, S, E), dO.double().view(B, S, E)
+    A = torch.bmm(fq, T(fk)).tril_()
+    d = A.sum(2, keepdim=True) + 1e-8
+    o = torch.bmm(A, v) / d
+    dn, dd = do / d, -(do * o).sum(2, keepdim=True) / d
+    G = (torch.bmm(dn, T(v)) + dd).tril_()
+    gq, gk = torch.bmm(G, fk) * fq.clamp(max=1), torch.bmm(T(G), fq) * fk.clamp(max=1)
+    # a score's error is (D / 8 + 16) 2^-24 of it (all terms positive), G's that
+    # of its terms' magnitudes; the sums over rows add (S / 8 + 16) 2^-24; the
+    # float angles of the rotation, up to S, 2^-24 S
+    e = (max(D, E) / 8 + S / 8 + 40 + (4 * S if api == "rope" else 0)) * 2.0 ** -24
+    H = (torch.bmm(dn.abs(), T(v.abs())) + (do * o).abs().sum(2, keepdim=True) / d).tril_() * e
+    lq, lk = torch.bmm(H, fk) * fq.clamp(max=1), torch.bmm(T(H), fq) * fk.clamp(max=1)
+    if api == "rope":
+        gq, gk = rot(gq, -1), rot(gk, -1)
+        lq, lk = (x.view(B, S, D // 2, 2).sum(3, keepdim=True).expand(-1, -1, -1, 2).reshape(B, S, D)
+                  for x in (lq, lk))
+    within(O, o.view(-1, E), (torch.bmm(A, v.abs()) / d).view(-1, E) * e * 2, "O")
+    within(den, d.view(-1), d.view(-1) * e, "den")
+    within(dV, torch.bmm(T(A), dn).view(-1, E), torch.bmm(T(A), dn.abs()).view(-1, E) * e * 2, "dV")
+    within(dQ, gq.reshape(-1, D), lq.view(-1, D) * 2, "dQ")
+    within(dK, gk.reshape(-1, D), lk.view(-1, D) * 2, "dK")
