@@ -182,6 +182,8 @@ __global__ __launch_bounds__(64 * NQ * NS) void mhabf_fwd_kernel(
         }
         const int k0 = kt * KT + 32 * ks;   // wave's first key
         if (k0 <= qw && qw < S) {           // else wholly above the diagonal
+            // products before the other waves' splitting ([2, 4096, 12, 64] 299 -> 287 us)
+            __builtin_amdgcn_s_setprio(1);
             const int row = 32 * ks + l32;
             f16 s = f16zero();
             b8 kh[NK];
@@ -263,6 +265,7 @@ __global__ __launch_bounds__(64 * NQ * NS) void mhabf_fwd_kernel(
                 }
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         if (DB && kt + 1 < nkt) {
             put(lds + ((kt & 1) ^ 1) * STAGE);
             if (kt + 2 < nkt)
@@ -368,7 +371,7 @@ static bool mhabf_ok(int S, int H, int Dh, const float* Q, const float* K, const
 //     rows there is nothing to share);
 //   more than two rounds and 256 rows or more: 128 queries a workgroup, so
 //     that a key tile is split once for twice the products ([2, 4096, 12, 64]
-//     293 / 402, [16, 384, 12, 64] 42.6 / 45.2, [16, 512, 12, 32] 30.3 / 37.7;
+//     287 / 402, [16, 384, 12, 64] 42.6 / 45.2, [16, 512, 12, 32] 30.3 / 37.7;
 //     shorter ones lose: [32, 128, 16, 64] 25.7 / 22.9);
 //   between one and two rounds mha.hip's paired jobs are the faster
 //     ([8, 256, 12, 64] 16.8 / 15.0).
@@ -718,10 +721,10 @@ static hipError_t bwd_go(const float* Q, const float* K, const float* V, const f
 //   heads past 64 columns: all ([4, 333, 10, 80] 56.3 / 111.6 us, [32, 64, 16,
 //     96] 50.6 / 58.5);
 //   33 to 64 columns, at most one 64-key tile a compute unit and 128 rows or
-//     more, or at most two and more than 256: one workgroup of four waves a
-//     unit, with room to split the next query tile beside the products of this
+//     more, or at most two and 384 rows: one workgroup of four waves a unit, with room to split the next query tile beside the products of this
 //     one ([2, 512, 8, 64] 45.0 / 50.8, [4, 333, 10, 40] 35.9 / 41.5, [8, 512,
-//     8, 64] 60.9 / 64.0; [3, 90, 12, 64] 18.0 / 17.8);
+//     8, 64] 60.9 / 64.0; [3, 90, 12, 64] 18.0 / 17.8, [5, 300, 16, 64] 39.7 /
+//     38.9);
 //   more tiles and 256 rows or more: two workgroups a unit, dS taking dO's
 //     place in LDS ([2, 4096, 12, 64] 816 / 1040, [16, 384, 12, 64] 99.7 /
 //     118.2; [32, 128, 16, 64] 56.1 / 52.9);
@@ -734,7 +737,7 @@ static int bwd_kind(int B, int S, int H, int Dh)
     if (Dh <= 32)
         return BF_NONE;
     if (tiles <= 2 * cus)
-        return S >= (tiles <= cus ? 128 : 257) ? BF_SHARED : BF_NONE;
+        return S >= (tiles <= cus ? 128 : 384) ? BF_SHARED : BF_NONE;
     return S >= 256 ? BF_LONG : BF_NONE;
 }
 
