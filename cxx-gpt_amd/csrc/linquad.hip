@@ -603,7 +603,8 @@ __global__ __launch_bounds__(256) void lin_qs_prod_kernel(const QsArgs a,
 // stages (three), were slower at every shape.  Kernel times, one wave a 16-row
 // unit -> tiles: 32 x S256, D = E = 512: gradients 54.8 -> 43.3 us, O 19.2 ->
 // 15.6; 32 x S384, 640: 156 -> 95.5, 50.8 -> 35.1; 8 x S256, 512: gradients
-// 18.9 -> 15.2.
+// 18.9 -> 15.2.  An infinity or NaN in a row of X meets the zero scores of the
+// rows before it in its 32-row step (of its 16-row block above).
 // ---------------------------------------------------------------------------
 template <int PHI, bool BWD>
 __global__ __launch_bounds__(256) void lin_qs_tile_kernel(const QsArgs a,

@@ -721,9 +721,10 @@ static hipError_t bwd_go(const float* Q, const float* K, const float* V, const f
 //   heads past 64 columns: all ([4, 333, 10, 80] 56.3 / 111.6 us, [32, 64, 16,
 //     96] 50.6 / 58.5);
 //   33 to 64 columns, at most one 64-key tile a compute unit and 128 rows or
-//     more, or at most two and 384 rows: one workgroup of four waves a unit, with room to split the next query tile beside the products of this
-//     one ([2, 512, 8, 64] 45.0 / 50.8, [4, 333, 10, 40] 35.9 / 41.5, [8, 512,
-//     8, 64] 60.9 / 64.0; [3, 90, 12, 64] 18.0 / 17.8, [5, 300, 16, 64] 39.7 /
+//     more, or at most two and 384 rows: one workgroup of four waves a unit,
+//     with room to split the next query tile beside the products of this one
+//     ([2, 512, 8, 64] 45.0 / 50.8, [4, 333, 10, 40] 35.9 / 41.5, [8, 512, 8,
+//     64] 60.9 / 64.0; [3, 90, 12, 64] 18.0 / 17.8, [5, 300, 16, 64] 39.7 /
 //     38.9);
 //   more tiles and 256 rows or more: two workgroups a unit, dS taking dO's
 //     place in LDS ([2, 4096, 12, 64] 816 / 1040, [16, 384, 12, 64] 99.7 /
